@@ -767,7 +767,9 @@ void prepare_tables(SamplerTables& t, const void* state, uint32_t n) {
 template <typename V>
 void launch_shots(const SampleArgs& a, const double* u, uint64_t shots, uint64_t* out, uint64_t first_index,
                   bool sorted, bool partial, hipStream_t stream) {
-    constexpr uint64_t kMaxGrid = uint64_t{1} << 30;
+    // A launch takes fewer than 2^32 threads.
+    constexpr uint64_t kMaxGrid = uint64_t{1} << 23;
+    static_assert(kMaxGrid * kThreads < uint64_t{1} << 32);
     for (uint64_t at = 0; at < shots; at += kMaxGrid) {
         const uint64_t count = std::min(shots - at, kMaxGrid);
         hipLaunchKernelGGL(shots_kernel<V>, dim3(static_cast<uint32_t>(count)), dim3(kThreads), 0, stream, a, u + at,

@@ -2,7 +2,7 @@
 it, the last basis if none does. Uniforms below 0 and far above the total, and
 states whose running sum turns infinite or NaN (a NaN exceeds nothing), in the
 single-launch form, in the table form with one and with several groups of
-blocks, sorted and unsorted."""
+blocks, sorted and unsorted; and more shots than one launch takes."""
 import numpy as np
 import pytest
 
@@ -52,3 +52,16 @@ def test_sums_that_are_not_finite(orc, hip, n, at, value):
     s[{"first": 0, "early": s.size // 100, "middle": s.size // 2 - 1, "last": s.size - 1}[at]] = value
     u = np.concatenate([np.random.default_rng(n).random(24), [-1.0, 0.0, 1e-9, 0.4999, 0.5001, 1.5]])
     _check(hip, orc, s, u)
+
+
+def test_more_shots_than_one_launch(orc, hip):
+    """2^23 shots a launch: the boundary falls inside a block's shots."""
+    n, shots = 15, (1 << 23) + 1000
+    s = random_state(n, 9)
+    u = np.sort(np.random.default_rng(3).random(shots))
+    d = hip.DeviceState(n)
+    d.upload(s)
+    got = d.sample(u).astype(np.int64)
+    d.free()
+    want = np.minimum(np.searchsorted(orc.cumulative(s), u, side="right"), s.size - 1)
+    assert np.array_equal(got, want)
