@@ -10,6 +10,10 @@ namespace mh {
 
 // Tile qubits of a wide pass: the smallest state it takes.
 constexpr uint32_t kWideTileBits = 12;
+// ... and the largest: a workgroup of 512 threads a tile, and a launch takes
+// fewer than 2^32 threads (a complex64 state of 35 qubits, 256 GiB, goes to the
+// per-group kernel, whose grid does not grow with it).
+constexpr uint32_t kWideQubits = 34;
 // Blocks of one pass at most: its arithmetic is by then many times the read
 // and write of the state that they share, and a run's monitor is asked between
 // passes.
@@ -19,7 +23,8 @@ constexpr uint32_t kWidePassBlocks = 16;
 constexpr uint64_t kWideTableBytes = uint64_t{16} << 20;
 
 // Whether a dense block of k qubits of an n-qubit state goes to a wide pass:
-// three to six qubits, except the complex64 blocks that the matrix cores take.
+// three to six qubits, except the complex64 blocks that the matrix cores take
+// and states beyond one launch.
 bool wide_applies(int32_t precision, uint32_t n, uint32_t k);
 
 // The lowest qubits, which every tile holds: runs of 128 bytes.

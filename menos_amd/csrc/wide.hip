@@ -39,6 +39,7 @@ constexpr uint32_t kOuts = (1u << kTileBits) / kThreads;  // outputs (and loaded
 constexpr uint32_t kThreadBits = 9;
 constexpr uint32_t kMaxK = 6;
 static_assert(kOuts == 8 && kThreads == 1u << kThreadBits);
+static_assert((uint64_t{1} << (kWideQubits - kTileBits)) * kThreads < uint64_t{1} << 32);
 
 template <typename R> struct Vec;
 template <> struct Vec<double> { using type = double2; };
@@ -220,7 +221,7 @@ __global__ void __launch_bounds__(kThreads, 4) wide_kernel(WideArgs args) {
 }  // namespace
 
 bool wide_applies(int32_t precision, uint32_t n, uint32_t k) {
-    return n >= kWideTileBits && k >= 3 && k <= (precision == MH_C128 ? kMaxK : 4);
+    return n >= kWideTileBits && n <= kWideQubits && k >= 3 && k <= (precision == MH_C128 ? kMaxK : 4);
 }
 
 uint64_t wide_low_mask(int32_t precision) { return precision == MH_C128 ? 7 : 15; }
@@ -353,8 +354,8 @@ void WidePasses::launch(void* state, uint32_t pass, hipStream_t stream) const {
     a.outer_mask = p.outer_mask;
     a.count = p.count;
     std::memcpy(a.tpos, p.tpos, sizeof(a.tpos));
+    if (d.n < kTileBits || d.n > kWideQubits) fail(MH_ERR_INTERNAL, "wide pass shape out of range");
     const uint32_t tiles = 1u << (d.n - kTileBits);
-    if (d.n - kTileBits > 30) fail(MH_ERR_INTERNAL, "wide pass shape out of range");
     if (d.precision == MH_C128)
         hipLaunchKernelGGL(wide_kernel<double>, dim3(tiles), dim3(kThreads), 0, stream, a);
     else
