@@ -31,7 +31,7 @@
 // Prediction only decides speed: every transfer is checked against the exact
 // running value before it is used.
 //
-// A state of at most 14 qubits takes one workgroup and one launch for all of it.
+// A state of at most 14 qubits takes one launch for all of it.
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -593,9 +593,14 @@ __device__ __forceinline__ uint64_t resolve(const StageShared& sh, uint32_t coun
     return none;
 }
 
-// Workgroup i is shot i's. Sorted uniforms: the first shot of a block takes
-// every shot of that block, the others' workgroups end; else each takes its
-// own. Every uniform gets the first index whose running sum exceeds it (one
+// Shots a workgroup takes from one reading of their block, at most.
+constexpr uint32_t kShare = 1024;
+
+// Workgroup i has shots [i * piece, (i + 1) * piece), piece a divisor of kShare
+// (1 unless they are sorted and all of the state's). Sorted uniforms: the first
+// shot of a block, and each whose number is a multiple of kShare, takes the
+// shots of its block up to the next such; the others leave theirs to it. Else
+// each takes its own. Every uniform gets the first index whose running sum exceeds it (one
 // below 0 index 0), else the last index; for one chunk of a state (`partial`, `first_index` the chunk's first index) one
 // that another chunk's sums exceed first is left alone. Comparisons are with
 // "at most", so that the searches hold where the sum turns NaN, which exceeds
@@ -606,72 +611,112 @@ __device__ __forceinline__ uint64_t resolve(const StageShared& sh, uint32_t coun
 // 4096 at 17; walking them with one thread per shot took 2.26 and 1.24.
 template <typename V>
 __global__ void __launch_bounds__(kThreads) shots_kernel(SampleArgs a, const double* u, uint64_t shots, uint64_t* out,
-                                                        uint64_t first_index, bool sorted, bool partial) {
+                                                        uint64_t first_index, bool sorted, bool partial,
+                                                        uint32_t piece) {
     __shared__ StageShared sh;
-    const uint64_t i = blockIdx.x;
     const uint32_t t = threadIdx.x;
-    const double x = u[i];
+    const uint64_t begin = uint64_t(blockIdx.x) * piece, end = min(begin + piece, shots);
     const bool opens = first_index == 0;  // nothing comes before this state (or chunk)
-    if (partial && (x >= a.cstart[a.blocks] || !(opens || x >= a.cstart[0]))) return;
-    // The first block whose end value is not at most x, kThreads pivots at a
-    // time.
-    uint32_t lo = 0, hi = a.blocks;  // the answer is in [lo, hi]
-    while (lo < hi) {
-        const uint32_t step = (hi - lo + kThreads - 1) / kThreads;
-        const uint64_t at = uint64_t(lo) + uint64_t(t + 1) * step - 1;  // the last block of the thread's share
-        const bool past = at < hi && x >= a.cstart[at + 1];
-        const uint32_t shares = static_cast<uint32_t>(__syncthreads_count(past));
-        const uint64_t begin = uint64_t(lo) + uint64_t(shares) * step;
-        const uint32_t limit = hi;
-        lo = static_cast<uint32_t>(min(begin, uint64_t{limit}));
-        hi = static_cast<uint32_t>(min(begin + step - 1, uint64_t{limit}));
-    }
-    if (lo == a.blocks) {
-        if (t == 0) out[i] = first_index + a.size - 1;
-        return;
-    }
-    const double c0 = a.cstart[lo], c1 = a.cstart[lo + 1];
-    // The block's first shot takes this one.
-    if (sorted && i > 0 && ((opens && lo == 0) || u[i - 1] >= c0)) return;
-    uint64_t count = 1;
-    if (sorted) {
-        count = 0;
-        for (uint32_t more = kThreads; more == kThreads;) {
-            const uint64_t at = i + count + t;
-            more = static_cast<uint32_t>(__syncthreads_count(at < shots && !(u[at] >= c1)));
-            count += more;
+    for (uint64_t i = begin; i < end;) {
+        const double x = u[i];
+        if (partial && (x >= a.cstart[a.blocks] || !(opens || x >= a.cstart[0]))) return;
+        // The first block whose end value is not at most x, kThreads pivots at a
+        // time.
+        uint32_t lo = 0, hi = a.blocks;  // the answer is in [lo, hi]
+        while (lo < hi) {
+            const uint32_t step = (hi - lo + kThreads - 1) / kThreads;
+            const uint64_t at = uint64_t(lo) + uint64_t(t + 1) * step - 1;  // the last block of the thread's share
+            const bool past = at < hi && x >= a.cstart[at + 1];
+            const uint32_t shares = static_cast<uint32_t>(__syncthreads_count(past));
+            const uint64_t from = uint64_t(lo) + uint64_t(shares) * step;
+            const uint32_t limit = hi;
+            lo = static_cast<uint32_t>(min(from, uint64_t{limit}));
+            hi = static_cast<uint32_t>(min(from + step - 1, uint64_t{limit}));
         }
-    }
-    const double last = u[i + count - 1];
-    const V* st = static_cast<const V*>(a.state);
-    const uint32_t stage = static_cast<uint32_t>(min(a.block, uint64_t{kStage}));
-    double c = c0;
-    for (uint64_t at = 0; at < a.block; at += stage) {
-        const uint64_t i0 = uint64_t(lo) * a.block + at;
-        load_stage(sh, st, i0, stage);
-        exact_stage(sh, stage, c);
-        c = sh.start[kThreads];
-        for (uint64_t j = t; j < count; j += kThreads) {
-            const double y = u[i + j];
-            // A NaN: an earlier stage's sums, if any, were at most y.
-            if ((at == 0 || y >= sh.start[0]) && !(y >= c)) {
-                const uint64_t hit = resolve(sh, stage, i0, y, UINT64_MAX);
-                if (hit != UINT64_MAX)
-                    out[i + j] = first_index + hit;
-                else if (!partial)
-                    out[i + j] = a.size - 1;
+        if (lo == a.blocks) {  // sorted: the later ones as well
+            for (uint64_t j = i + t; j < end; j += kThreads) out[j] = first_index + a.size - 1;
+            return;
+        }
+        const double c0 = a.cstart[lo], c1 = a.cstart[lo + 1];
+        const bool takes = !sorted || i % kShare == 0 || !((opens && lo == 0) || u[i - 1] >= c0);
+        uint64_t count = 1;
+        if (sorted) {
+            const uint64_t limit = takes ? min(shots, (i / kShare + 1) * kShare) : end;
+            count = 0;
+            for (uint32_t more = kThreads; more == kThreads;) {
+                const uint64_t at = i + count + t;
+                more = static_cast<uint32_t>(__syncthreads_count(at < limit && !(u[at] >= c1)));
+                count += more;
             }
         }
-        if (!(last >= c)) break;
-        __syncthreads();
+        if (takes) {
+            const double last = u[i + count - 1];
+            const V* st = static_cast<const V*>(a.state);
+            const uint32_t stage = static_cast<uint32_t>(min(a.block, uint64_t{kStage}));
+            double c = c0;
+            for (uint64_t at = 0; at < a.block; at += stage) {
+                const uint64_t i0 = uint64_t(lo) * a.block + at;
+                load_stage(sh, st, i0, stage);
+                exact_stage(sh, stage, c);
+                c = sh.start[kThreads];
+                for (uint64_t j = t; j < count; j += kThreads) {
+                    const double y = u[i + j];
+                    // A NaN: an earlier stage's sums, if any, were at most y.
+                    if ((at == 0 || y >= sh.start[0]) && !(y >= c)) {
+                        const uint64_t hit = resolve(sh, stage, i0, y, UINT64_MAX);
+                        if (hit != UINT64_MAX)
+                            out[i + j] = first_index + hit;
+                        else if (!partial)
+                            out[i + j] = a.size - 1;
+                    }
+                }
+                __syncthreads();
+                if (!(last >= c)) break;
+            }
+        }
+        i += count;
     }
 }
 
-// A small state's shots (any order) by one workgroup, stage by stage.
+// A thread per shot, in any order: its block by bisection, then plain adds from
+// the block's start (bound by their latency, so for many shots only).
+template <typename V>
+__global__ void __launch_bounds__(kThreads) shots_walk_kernel(SampleArgs a, const double* u, uint64_t shots,
+                                                             uint64_t* out) {
+    const uint64_t t = uint64_t(blockIdx.x) * kThreads + threadIdx.x;
+    if (t >= shots) return;
+    const double x = u[t];
+    uint32_t lo = 0, hi = a.blocks;  // the first block whose end value is not at most x
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (!(x >= a.cstart[mid + 1]))
+            hi = mid;
+        else
+            lo = mid + 1;
+    }
+    uint64_t hit = a.size - 1;
+    if (lo < a.blocks) {
+        const V* st = static_cast<const V*>(a.state);
+        const uint64_t i0 = uint64_t(lo) * a.block;
+        double c = a.cstart[lo];
+        for (uint64_t i = 0; i < a.block; ++i) {
+            c = c + prob(st, i0 + i);
+            if (x < c) {
+                hit = i0 + i;
+                break;
+            }
+        }
+    }
+    out[t] = hit;
+}
+
+// A small state's shots (any order), kShare of them a workgroup, each stage by
+// stage.
 template <typename V>
 __global__ void __launch_bounds__(kThreads) small_shots_kernel(const V* st, uint32_t size, const double* u,
                                                               uint64_t shots, uint64_t* out) {
     __shared__ StageShared sh;
+    const uint64_t begin = uint64_t(blockIdx.x) * kShare, last = min(begin + kShare, shots);
     double c = 0.0;
     for (uint32_t i0 = 0; i0 < size; i0 += kStage) {
         const uint32_t count = min(size - i0, kStage);
@@ -679,7 +724,7 @@ __global__ void __launch_bounds__(kThreads) small_shots_kernel(const V* st, uint
         exact_stage(sh, count, c);
         const bool end = i0 + count == size;
         c = sh.start[kThreads];
-        for (uint64_t j = threadIdx.x; j < shots; j += kThreads) {
+        for (uint64_t j = begin + threadIdx.x; j < last; j += kThreads) {
             const double y = u[j];
             if ((i0 == 0 || y >= sh.start[0]) && !(y >= c))
                 out[j] = resolve(sh, count, i0, y, size - 1);
@@ -763,17 +808,71 @@ void prepare_tables(SamplerTables& t, const void* state, uint32_t n) {
     launch_tables<V>(t.a, streams().main);
 }
 
+// States sampled without tables, in one launch: eight stages. Whole calls, this
+// form against the tables': 10 qubits and 100 shots 54 against 124 us, 14 qubits
+// and 1000 shots 110 against 175, 15 qubits 174 against 176. All of a state's
+// shots by one workgroup took 14.4 ms for 2,000,000 at 10 qubits, kShare a
+// workgroup 2.3.
+constexpr uint32_t kSmallQubits = 14;
+
+// Draws from a kept state of that size take this form too if it is one stage or
+// there are many of them (12 qubits, 1000 and 10,000 draws: 78 and 90 us, 78 and
+// 283 from the tables; 14 qubits 147 and 168, 73 and 184).
+constexpr uint64_t kSmallDraws = 4096;
+
+// Sorted shots go to about this many workgroups or more, up to kMostPiece of
+// them each (2,000,000 shots of 17 and 27 qubits, ms: 4096 workgroups 2.6 and
+// 6.9, 16384 2.9 and 5.3, 65536 3.4 and 6.3, one a shot 4.4 and 7.5).
+constexpr uint64_t kPieces = 16384;
+constexpr uint32_t kMostPiece = 256;
+static_assert(kShare % kMostPiece == 0);
+
+// Of so many shots in no order each walks its block by itself where the state
+// stays in the caches: a workgroup a shot reads the block for that one alone
+// (10,000, 100,000 and 2,000,000 draws: 16 qubits 0.33, 0.46 and 5.9 ms walked,
+// 0.15, 0.94 and 17 so; 21 qubits, with longer blocks, 1.4, 1.6 and 17, 0.24, 1.7
+// and 32; 23 qubits 1.6, 2.1 and 39, 0.21, 1.6 and 30).
+constexpr uint32_t kWalkQubits = 22;
+bool walked(const SampleArgs& a, uint64_t shots) {
+    return a.size <= (uint64_t{1} << kWalkQubits) && shots > (a.size <= (uint64_t{1} << kSmallBlockQubits) ? 1u << 15 : 1u << 16);
+}
+
+// A launch takes fewer than 2^32 threads.
+constexpr uint64_t kMaxGrid = uint64_t{1} << 23;
+static_assert(kMaxGrid * kThreads < uint64_t{1} << 32);
+
 // Queues the shots of a state (or chunk) whose tables are ready.
 template <typename V>
 void launch_shots(const SampleArgs& a, const double* u, uint64_t shots, uint64_t* out, uint64_t first_index,
                   bool sorted, bool partial, hipStream_t stream) {
-    // A launch takes fewer than 2^32 threads.
-    constexpr uint64_t kMaxGrid = uint64_t{1} << 23;
-    static_assert(kMaxGrid * kThreads < uint64_t{1} << 32);
-    for (uint64_t at = 0; at < shots; at += kMaxGrid) {
-        const uint64_t count = std::min(shots - at, kMaxGrid);
-        hipLaunchKernelGGL(shots_kernel<V>, dim3(static_cast<uint32_t>(count)), dim3(kThreads), 0, stream, a, u + at,
-                           count, out + at, first_index, sorted, partial);
+    uint32_t piece = 1;
+    if (sorted && !partial)
+        while (piece < kMostPiece && shots / (2 * piece) >= kPieces) piece *= 2;
+    for (uint64_t at = 0; at < shots; at += kMaxGrid * piece) {
+        const uint64_t count = std::min(shots - at, kMaxGrid * piece);
+        hipLaunchKernelGGL(shots_kernel<V>, dim3(static_cast<uint32_t>((count + piece - 1) / piece)), dim3(kThreads), 0,
+                           stream, a, u + at, count, out + at, first_index, sorted, partial, piece);
+        MH_HIP(hipGetLastError());
+    }
+}
+
+template <typename V>
+void launch_walks(const SampleArgs& a, const double* u, uint64_t shots, uint64_t* out, hipStream_t stream) {
+    for (uint64_t at = 0; at < shots; at += kMaxGrid * kThreads) {
+        const uint64_t count = std::min(shots - at, kMaxGrid * kThreads);
+        hipLaunchKernelGGL(shots_walk_kernel<V>, dim3(static_cast<uint32_t>((count + kThreads - 1) / kThreads)),
+                           dim3(kThreads), 0, stream, a, u + at, count, out + at);
+        MH_HIP(hipGetLastError());
+    }
+}
+
+template <typename V>
+void launch_small_shots(const V* state, uint32_t size, const double* u, uint64_t shots, uint64_t* out,
+                        hipStream_t stream) {
+    for (uint64_t at = 0; at < shots; at += kMaxGrid * kShare) {
+        const uint64_t count = std::min(shots - at, kMaxGrid * kShare);
+        hipLaunchKernelGGL(small_shots_kernel<V>, dim3(static_cast<uint32_t>((count + kShare - 1) / kShare)),
+                           dim3(kThreads), 0, stream, state, size, u + at, count, out + at);
         MH_HIP(hipGetLastError());
     }
 }
@@ -796,25 +895,23 @@ void draw_basis(const SampleArgs& a, const double* uniforms, uint64_t count, uin
     if (count == 0) return;
     context();
     ShotBuffers shots(uniforms, count);
-    launch_shots<V>(a, shots.u, count, shots.out, 0, std::is_sorted(uniforms, uniforms + count), false, streams().main);
+    const bool sorted = std::is_sorted(uniforms, uniforms + count);
+    if (a.size <= kStage || (a.size <= (uint64_t{1} << kSmallQubits) && count >= kSmallDraws))
+        launch_small_shots(static_cast<const V*>(a.state), static_cast<uint32_t>(a.size), shots.u, count, shots.out,
+                           streams().main);
+    else if (!sorted && walked(a, count))
+        launch_walks<V>(a, shots.u, count, shots.out, streams().main);
+    else
+        launch_shots<V>(a, shots.u, count, shots.out, 0, sorted, false, streams().main);
     download(basis_out, shots.out, count * sizeof(uint64_t));
 }
 
-// States one workgroup samples in one launch: eight stages. Whole calls, this
-// form against the tables': 10 qubits and 100 shots 54 against 124 us, 14
-// qubits and 1000 shots 127 against 175, 15 qubits 174 against 176; 12 qubits
-// and 5000 shots 151 against 216, 16,384 shots 302 against 322.
-constexpr uint32_t kSmallQubits = 14;
-constexpr uint64_t kSmallShots = 16384;
-
 template <typename V>
 void run_sampler(const void* state, uint32_t n, const double* sorted_u, uint64_t shots, uint64_t* basis_out) {
-    if (n <= kSmallQubits && shots <= kSmallShots) {
+    if (n <= kSmallQubits) {
         context();
         ShotBuffers io(sorted_u, shots);
-        hipLaunchKernelGGL(small_shots_kernel<V>, dim3(1), dim3(kThreads), 0, streams().main,
-                           static_cast<const V*>(state), 1u << n, static_cast<const double*>(io.u), shots, io.out);
-        MH_HIP(hipGetLastError());
+        launch_small_shots(static_cast<const V*>(state), 1u << n, io.u, shots, io.out, streams().main);
         download(basis_out, io.out, shots * sizeof(uint64_t));
         return;
     }

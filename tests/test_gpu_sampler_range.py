@@ -2,7 +2,8 @@
 it, the last basis if none does. Uniforms below 0 and far above the total, and
 states whose running sum turns infinite or NaN (a NaN exceeds nothing), in the
 single-launch form, in the table form with one and with several groups of
-blocks, sorted and unsorted; and more shots than one launch takes."""
+blocks, sorted and unsorted; and more shots than one
+launch, one workgroup or one reading of a block takes."""
 import numpy as np
 import pytest
 
@@ -65,3 +66,36 @@ def test_more_shots_than_one_launch(orc, hip):
     d.free()
     want = np.minimum(np.searchsorted(orc.cumulative(s), u, side="right"), s.size - 1)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("n,shots", [(3, 1024), (3, 1025), (9, 50000), (14, 4097), (14, 40000), (15, 1023), (15, 70001),
+                                     (17, 300000), (21, 100000)])
+def test_many_shots(orc, hip, n, shots):
+    """Both sides of the shots that a workgroup takes and of the forms for many
+    in no order, half of them on a few bases, with values below 0 and beyond
+    the total among them."""
+    s = random_state(n, n + 7)
+    s[s.size // 2:] *= 1e-3
+    cum = orc.cumulative(s)
+    rng = np.random.default_rng(shots)
+    u = np.concatenate([rng.random(shots // 2) * cum[-1], 0.3 + 1e-4 * rng.random(shots - shots // 2 - 20),
+                        -rng.random(10), cum[-1] + rng.random(10)])
+    want = np.minimum(np.searchsorted(cum, u, side="right"), s.size - 1)
+    order = np.argsort(u, kind="stable")
+    d = hip.DeviceState(n)
+    d.upload(s)
+    assert np.array_equal(d.sample(u[order]).astype(np.int64), want[order])
+    assert np.array_equal(d.sample_unsorted(u).astype(np.int64), want)
+    d.free()
+
+
+@pytest.mark.parametrize("n,draws", [(10, 1), (11, 5000), (12, 4095), (12, 4096), (14, 1), (15, 32768), (15, 32769),
+                                     (20, 40000), (21, 65536), (22, 65537), (23, 70000)])
+def test_draws_in_no_order(orc, hip, n, draws):
+    from menos_amd import workloads as W
+    r = hip.HipDenseEngine().execute(W.random_circuit(n, 3, n), statevector=True, region_sampler=True)
+    u = np.random.default_rng(draws).random(draws)
+    cum = orc.cumulative(r.statevector)
+    with r.region_sampler as s:
+        assert np.array_equal(s.draw(u).astype(np.int64),
+                              np.minimum(np.searchsorted(cum, u, side="right"), cum.size - 1))
