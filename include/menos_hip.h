@@ -497,9 +497,13 @@ int mh_batch_execute(const mh_batch_request* request, mh_batch_result* result);
  * mh_batch_graph_update takes new parameters for the same circuits (same
  * opcodes, qubits and parameter counts) and global phases (null: 0): block
  * matrices and pass programs are rebuilt on host threads and the new matrix
- * table is staged for the next run. A circuit whose structure differs, or
- * whose new matrices change its pass program (an entry that becomes or stops
- * being exactly 0 or +-1), is refused with MH_ERR_INVALID and nothing changes.
+ * table is staged for the next run (parameters such as a rotation by exactly
+ * 0, after which a block needs more or fewer products, may have the graph
+ * captured again). A circuit whose structure differs, or in which the new
+ * matrices take a block to another class, is refused with MH_ERR_INVALID and
+ * nothing changes: a block that becomes or stops being diagonal, a diagonal of
+ * signs (or changes those), controlled by one of its qubits or a controlled
+ * NOT, or a 1-qubit block whose first entry becomes or stops being real.
  * mh_batch_graph_run replays the graph once and writes the terms (2 doubles
  * per term, term order) into result->expectation_terms; it fills rounds,
  * launches (those the graph holds), the last update's plan and compile

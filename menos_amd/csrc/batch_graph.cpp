@@ -17,12 +17,18 @@
 //   terms -> pinned staging (copy node)
 //
 // A parameter update rebuilds the block matrices and pass programs on host
-// threads and, when every circuit's program keeps its shape (same passes, ops,
-// sign terms and launch lists: only matrix entries differ), writes the new
-// matrix table into the pinned staging the graph copies from. A run is one graph
-// launch. Results are the same kernels' as mh_batch_execute's, so terms equal it
-// bit for bit.
+// threads and writes the new matrix table into the pinned staging the graph
+// copies from. How a block runs depends on its matrix (a real one leaves out its
+// zero parts), so the program is built for the widest form that each block has
+// had: parameters that need a narrower one (a rotation by exactly 0) run in it,
+// and the first that need a wider one have the graph captured again. Only
+// parameters that take a block to another class (window.h) are refused: the
+// block becomes or stops being diagonal, controlled, a controlled NOT, or a
+// diagonal of signs, or the first entry of a 1-qubit block real. A run is one
+// graph launch. Results are the same kernels' as mh_batch_execute's, so terms
+// equal it bit for bit.
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstring>
 #include <memory>
@@ -111,6 +117,31 @@ struct Structure {
 }  // namespace
 }  // namespace mh
 
+namespace mh {
+namespace {
+
+// A program, its tables on the device and the graph that runs it.
+struct Captured {
+    BatchProgram program;
+    std::unique_ptr<EarlyReductions> reductions;
+    DeviceBuffer bundles, ops, terms, mats, args, groups;
+    Pinned pinned_mats;
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    uint32_t launches = 0;
+
+    Captured() = default;
+    Captured(const Captured&) = delete;
+    Captured& operator=(const Captured&) = delete;
+    ~Captured() {
+        if (exec) (void)hipGraphExecDestroy(exec);
+        if (graph) (void)hipGraphDestroy(graph);
+    }
+};
+
+}  // namespace
+}  // namespace mh
+
 struct mh_batch_graph {
     int32_t precision = MH_C128;
     int32_t fusion = MH_FUSE_CONTAINMENT;
@@ -122,23 +153,16 @@ struct mh_batch_graph {
     uint32_t total_terms = 0;
     std::vector<mh::Structure> structure;
     std::vector<std::vector<mh::Block>> blocks;
+    std::vector<std::vector<mh::BlockForm>> forms;  // of each block, the widest so far
     std::vector<mh::BatchItem> items;
-    mh::BatchProgram program;
-    std::unique_ptr<mh::EarlyReductions> reductions;
     std::vector<uint32_t> term_offsets;
+    std::vector<uint64_t> x_masks, z_masks;
     // Device residency.
-    mh::DeviceBuffer arena, bundles, ops, terms, mats, args, groups, dterms;
+    mh::DeviceBuffer arena, dterms;
     uint64_t arena_bytes = 0;
-    mh::Pinned pinned_mats, pinned_terms;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    uint32_t launches = 0;
+    mh::Pinned pinned_terms;
+    std::unique_ptr<mh::Captured> captured;
     double plan_seconds = 0, compile_seconds = 0;
-
-    ~mh_batch_graph() {
-        if (exec) (void)hipGraphExecDestroy(exec);
-        if (graph) (void)hipGraphDestroy(graph);
-    }
 };
 
 namespace mh {
@@ -157,6 +181,7 @@ void plan_all(mh_batch_graph& g, const mh_circuit* circuits) {
         validate_circuit(&circuits[i]);
         const CircuitView cv{&circuits[i]};
         g.blocks[i] = build_blocks(cv, plan_fusion(cv, g.fusion, g.fusion_width));
+        g.forms[i] = classify(g.blocks[i], g.precision);
     });
     g.plan_seconds = seconds_since(t0);
 }
@@ -171,7 +196,8 @@ void set_phases(std::vector<BatchItem>& items, const double* global_phases) {
     }
 }
 
-// Everything on the main stream. A graph captured over several streams (the
+// Uploads a program's tables and captures its launches, everything on the main
+// stream. A graph captured over several streams (the
 // kernel streams forked off the main stream and joined back) kept the device
 // memory its kernels used referenced after the graph and its executable were
 // destroyed (measured on ROCm 7.2: hipFree returned success and the memory did
@@ -179,28 +205,58 @@ void set_phases(std::vector<BatchItem>& items, const double* global_phases) {
 // stream, the memory returns. One launch group at a time on one stream costs
 // the default schedule nothing (it has one launch group), and the reduction
 // buckets follow the launch that finishes their states.
-void capture(mh_batch_graph& g) {
+std::unique_ptr<Captured> capture(const mh_batch_graph& g, const std::vector<BatchItem>& items, BatchProgram&& program) {
     context();
+    auto c = std::make_unique<Captured>();
+    c->program = std::move(program);
+    auto table = [](DeviceBuffer& d, const std::vector<unsigned char>& src) {
+        d = DeviceBuffer(src.size());
+        upload(d.get(), src.data(), src.size());
+    };
+    table(c->bundles, c->program.bundles());
+    table(c->ops, c->program.ops());
+    table(c->terms, c->program.terms());
+    table(c->args, c->program.args());
+    table(c->groups, c->program.groups());
+    c->mats = DeviceBuffer(c->program.mats().size());
+    c->pinned_mats = Pinned(c->program.mats().size());
+    std::memcpy(c->pinned_mats.get(), c->program.mats().data(), c->program.mats().size());
+    if (g.total_terms > 0) {
+        std::vector<ExpectationItem> terms(g.count);
+        for (uint32_t i = 0; i < g.count; ++i) {
+            ExpectationItem& e = terms[i];
+            e.state = items[i].state;
+            e.n = items[i].n;
+            e.terms = g.term_offsets[i + 1] - g.term_offsets[i];
+            e.x = g.x_masks.data() + g.term_offsets[i];
+            e.z = g.z_masks.data() + g.term_offsets[i];
+            e.out_index = g.term_offsets[i];
+        }
+        c->reductions = std::make_unique<EarlyReductions>(g.precision, c->program, terms, g.dterms.as<double>(), streams().main);
+        c->reductions->upload(streams().copy, false);
+        MH_HIP(hipStreamSynchronize(streams().copy));
+    }
+    synchronize();
     const hipStream_t main = streams().main;
     BatchSchedule one = g.schedule;
     one.kernel_streams = 1;
     BatchDeviceTables dev;
-    dev.bundles = g.bundles.as<uint32_t>();
-    dev.ops = static_cast<const WOp*>(g.ops.get());
-    dev.terms = static_cast<const SignTerm*>(g.terms.get());
-    dev.mats = g.mats.get();
-    dev.args = static_cast<const WBatchArgs*>(g.args.get());
-    dev.groups = g.groups.as<uint32_t>();
+    dev.bundles = c->bundles.as<uint32_t>();
+    dev.ops = static_cast<const WOp*>(c->ops.get());
+    dev.terms = static_cast<const SignTerm*>(c->terms.get());
+    dev.mats = c->mats.get();
+    dev.args = static_cast<const WBatchArgs*>(c->args.get());
+    dev.groups = c->groups.as<uint32_t>();
     MH_HIP(hipStreamBeginCapture(main, hipStreamCaptureModeThreadLocal));
     try {
-        MH_HIP(hipMemcpyAsync(g.mats.get(), g.pinned_mats.get(), g.program.mats().size(), hipMemcpyHostToDevice, main));
+        MH_HIP(hipMemcpyAsync(c->mats.get(), c->pinned_mats.get(), c->program.mats().size(), hipMemcpyHostToDevice, main));
         AfterLaunch after;
-        if (g.reductions) after = [&](const BatchLaunch& l, hipStream_t s) { g.reductions->after(l, s); };
-        g.launches = issue_batch_program(g.program, g.items.data(), dev, one, 0, after);
-        if (g.reductions) {
-            g.reductions->flush({main});
+        if (c->reductions) after = [&](const BatchLaunch& l, hipStream_t s) { c->reductions->after(l, s); };
+        c->launches = issue_batch_program(c->program, items.data(), dev, one, 0, after);
+        if (c->reductions) {
+            c->reductions->flush({main});
             MH_HIP(hipMemcpyAsync(g.pinned_terms.get(), g.dterms.get(), g.dterms.bytes(), hipMemcpyDeviceToHost, main));
-            g.launches += g.reductions->launches();
+            c->launches += c->reductions->launches();
         }
     } catch (...) {
         hipGraph_t partial = nullptr;
@@ -208,8 +264,9 @@ void capture(mh_batch_graph& g) {
         if (partial) (void)hipGraphDestroy(partial);
         throw;
     }
-    MH_HIP(hipStreamEndCapture(main, &g.graph));
-    MH_HIP(hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
+    MH_HIP(hipStreamEndCapture(main, &c->graph));
+    MH_HIP(hipGraphInstantiate(&c->exec, c->graph, nullptr, nullptr, 0));
+    return c;
 }
 
 }  // namespace
@@ -218,7 +275,8 @@ void capture(mh_batch_graph& g) {
 namespace mh {
 namespace {
 // New parameters (circuits of the captured structure) into the staged matrix
-// table; refuses a change of any pass program.
+// table, or into a new graph where some block needs a wider form; refuses a
+// change of a block's class.
 void update_blocks(mh_batch_graph& g, const mh_circuit* circuits, const double* global_phases);
 }  // namespace
 }  // namespace mh
@@ -252,6 +310,7 @@ int mh_batch_graph_create(const mh_batch_request* req, mh_batch_graph** out) {
         const uint32_t width = window_width(req->precision);
         g->structure.resize(g->count);
         g->blocks.resize(g->count);
+        g->forms.resize(g->count);
         g->items.resize(g->count);
         g->term_offsets.assign(req->term_offsets, req->term_offsets + g->count + 1);
         uint64_t arena_bytes = 0;
@@ -277,57 +336,30 @@ int mh_batch_graph_create(const mh_batch_request* req, mh_batch_graph** out) {
         g->arena_bytes = arena_bytes;
         g->arena = DeviceBuffer(arena_bytes);
         unsigned char* base = static_cast<unsigned char*>(g->arena.get());
-        std::vector<ExpectationItem> exp_items(g->count);
-        bool any_terms = false;
+        if (g->total_terms > 0) {
+            g->x_masks.assign(req->x_masks, req->x_masks + g->total_terms);
+            g->z_masks.assign(req->z_masks, req->z_masks + g->total_terms);
+            g->dterms = DeviceBuffer(uint64_t(g->total_terms) * 2 * sizeof(double));
+            g->pinned_terms = Pinned(g->dterms.bytes());
+        }
         uint64_t at = 0;
         for (uint32_t i = 0; i < g->count; ++i) {
             BatchItem& it = g->items[i];
             it.state = base + at;
             it.n = req->circuits[i].num_qubits;
             it.blocks = &g->blocks[i];
+            it.forms = &g->forms[i];
             it.max_cost = req->max_pass_cost;
-            const uint32_t nt = req->term_offsets[i + 1] - req->term_offsets[i];
-            if (nt > 0) {
-                ExpectationItem& e = exp_items[i];
-                e.state = it.state;
-                e.n = it.n;
-                e.terms = nt;
-                e.x = req->x_masks + req->term_offsets[i];
-                e.z = req->z_masks + req->term_offsets[i];
-                e.out_index = req->term_offsets[i];
-                any_terms = true;
-            }
             at += round_state_bytes(it.n, req->precision);
         }
         set_phases(g->items, req->global_phases);
         const auto c0 = std::chrono::steady_clock::now();
-        g->program = compile_batch_program(req->precision, g->items.data(), g->count, g->threads, g->schedule);
+        BatchProgram program = compile_batch_program(req->precision, g->items.data(), g->count, g->threads, g->schedule);
         g->compile_seconds = seconds_since(c0);
-        if (g->program.has_generic() || g->program.needs_initialisation())
+        if (program.has_generic() || program.needs_initialisation())
             fail(MH_ERR_INVALID, "a captured batch takes circuits with at least one gate and blocks of at most 2 "
                                  "qubits (dense) or diagonal blocks");
-        auto table = [](DeviceBuffer& d, const std::vector<unsigned char>& src) {
-            d = DeviceBuffer(src.size());
-            upload(d.get(), src.data(), src.size());
-        };
-        table(g->bundles, g->program.bundles());
-        table(g->ops, g->program.ops());
-        table(g->terms, g->program.terms());
-        table(g->args, g->program.args());
-        table(g->groups, g->program.groups());
-        g->mats = DeviceBuffer(g->program.mats().size());
-        g->pinned_mats = Pinned(g->program.mats().size());
-        std::memcpy(g->pinned_mats.get(), g->program.mats().data(), g->program.mats().size());
-        if (any_terms) {
-            g->dterms = DeviceBuffer(uint64_t(g->total_terms) * 2 * sizeof(double));
-            g->reductions = std::make_unique<EarlyReductions>(req->precision, g->program, exp_items,
-                                                              g->dterms.as<double>(), streams().main);
-            g->reductions->upload(streams().copy, false);
-            MH_HIP(hipStreamSynchronize(streams().copy));
-            g->pinned_terms = Pinned(g->dterms.bytes());
-        }
-        synchronize();
-        capture(*g);
+        g->captured = capture(*g, g->items, std::move(program));
         *out = g.release();
     });
 }
@@ -373,31 +405,73 @@ int mh_batch_graph_param_count(const mh_batch_graph* g, uint64_t* out) {
 namespace mh {
 namespace {
 
+// Whether two diagonals of signs have the same ones.
+bool same_signs(const Block& a, const Block& b) {
+    const std::size_t dim = std::size_t{1} << a.operands.size();
+    for (std::size_t e = 0; e < dim; ++e)
+        if (a.matrix[e * dim + e].real() != b.matrix[e * dim + e].real()) return false;
+    return true;
+}
+
 void update_blocks(mh_batch_graph& gr, const mh_circuit* circuits, const double* global_phases) {
     mh_batch_graph* g = &gr;
-    {
-        std::vector<std::vector<Block>> fresh(g->count);
-        const auto t0 = clock_type::now();
-        parallel_for(g->count, g->threads, [&](std::size_t i) {
-            validate_circuit(&circuits[i]);
-            const CircuitView cv{&circuits[i]};
-            fresh[i] = build_blocks(cv, plan_fusion(cv, g->fusion, g->fusion_width));
-        });
-        g->plan_seconds = seconds_since(t0);
-        std::vector<BatchItem> items = g->items;
-        for (uint32_t i = 0; i < g->count; ++i) items[i].blocks = &fresh[i];
-        set_phases(items, global_phases);
-        const auto c0 = clock_type::now();
-        BatchProgram prog = compile_batch_program(g->precision, items.data(), g->count, g->threads, g->schedule);
-        g->compile_seconds = seconds_since(c0);
-        if (!prog.same_shape(g->program))
-            fail(MH_ERR_INVALID, "the new parameters change a pass program (a matrix entry became or stopped being "
-                                 "exactly zero or +-1); create a new captured batch for them");
-        std::memcpy(g->pinned_mats.get(), prog.mats().data(), prog.mats().size());
-        g->blocks = std::move(fresh);
-        g->items = std::move(items);
-        for (uint32_t i = 0; i < g->count; ++i) g->items[i].blocks = &g->blocks[i];
-        g->program = std::move(prog);
+    std::vector<std::vector<Block>> fresh(g->count);
+    std::vector<std::vector<BlockForm>> wider(g->count);  // a circuit's forms, where one got wider
+    std::atomic<bool> refused{false}, again{false};
+    const auto t0 = clock_type::now();
+    parallel_for(g->count, g->threads, [&](std::size_t i) {
+        validate_circuit(&circuits[i]);
+        const CircuitView cv{&circuits[i]};
+        fresh[i] = build_blocks(cv, plan_fusion(cv, g->fusion, g->fusion_width));
+        const std::vector<Block>& before = g->blocks[i];
+        bool ok = fresh[i].size() == before.size();
+        for (std::size_t b = 0; ok && b < before.size(); ++b) ok = fresh[i][b].operands == before[b].operands;
+        if (!ok) {
+            refused = true;
+            return;
+        }
+        const std::vector<BlockForm> forms = classify(fresh[i], g->precision);
+        for (std::size_t b = 0; b < before.size(); ++b) {
+            BlockForm f = wider[i].empty() ? g->forms[i][b] : wider[i][b];
+            if (!join_form(f, forms[b], before[b].operands) ||
+                (f.kind == BlockForm::kSign && !same_signs(fresh[i][b], before[b]))) {
+                refused = true;
+                return;
+            }
+            if (f == g->forms[i][b]) continue;
+            if (wider[i].empty()) wider[i] = g->forms[i];
+            wider[i][b] = f;
+            again = true;
+        }
+    });
+    g->plan_seconds = seconds_since(t0);
+    const char* const changed =
+        "the new parameters change a pass program (a matrix entry became or stopped being "
+        "exactly zero or +-1); create a new captured batch for them";
+    if (refused) fail(MH_ERR_INVALID, changed);
+    std::vector<BatchItem> items = g->items;
+    for (uint32_t i = 0; i < g->count; ++i) {
+        items[i].blocks = &fresh[i];
+        if (!wider[i].empty()) items[i].forms = &wider[i];
+    }
+    set_phases(items, global_phases);
+    const auto c0 = clock_type::now();
+    BatchProgram prog = compile_batch_program(g->precision, items.data(), g->count, g->threads, g->schedule);
+    if (again) {
+        g->captured = capture(*g, items, std::move(prog));
+    } else {
+        if (!prog.same_shape(g->captured->program)) fail(MH_ERR_INVALID, changed);
+        std::memcpy(g->captured->pinned_mats.get(), prog.mats().data(), prog.mats().size());
+        g->captured->program = std::move(prog);
+    }
+    g->compile_seconds = seconds_since(c0);
+    g->blocks = std::move(fresh);
+    for (uint32_t i = 0; i < g->count; ++i)
+        if (!wider[i].empty()) g->forms[i] = std::move(wider[i]);
+    g->items = std::move(items);
+    for (uint32_t i = 0; i < g->count; ++i) {
+        g->items[i].blocks = &g->blocks[i];
+        g->items[i].forms = &g->forms[i];
     }
 }
 
@@ -412,15 +486,15 @@ int mh_batch_graph_run(mh_batch_graph* g, mh_batch_result* res) {
         if (g->total_terms > 0 && res->expectation_terms == nullptr) fail(MH_ERR_INVALID, "no term output");
         const auto t0 = clock_type::now();
         context();
-        MH_HIP(hipGraphLaunch(g->exec, streams().main));
+        MH_HIP(hipGraphLaunch(g->captured->exec, streams().main));
         synchronize();
-        if (g->reductions)
+        if (g->total_terms > 0)
             std::memcpy(res->expectation_terms, g->pinned_terms.get(), uint64_t(g->total_terms) * 2 * sizeof(double));
         const double secs = seconds_since(t0);
         if (res->completion_seconds)
             for (uint32_t i = 0; i < g->count; ++i) res->completion_seconds[i] = secs;
         res->rounds = 1;
-        res->launches = g->launches;
+        res->launches = g->captured->launches;
         res->plan_seconds = g->plan_seconds;
         res->compile_seconds = g->compile_seconds;
         res->device_seconds = secs;
