@@ -26,6 +26,7 @@ struct BatchLaunch {
     uint32_t total_groups = 0;
     bool pairs = false;
     uint32_t group = 0, pass = 0;
+    uint32_t wave_bits = 0;  // of its widest window: the workgroups have 2^wave_bits wavefronts
 };
 
 // The tables of a program in device memory.
