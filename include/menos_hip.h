@@ -231,7 +231,10 @@ typedef enum mh_fusion {
  * every block, src/engines/dense/fused_block.h:96-99). mh_engine_execute calls
  * it after each HBM pass, on the calling thread, with the number of passes
  * completed so far (from 1): there the state holds every block of those passes
- * and nothing has been handed to the caller. The reference abandons by
+ * and nothing has been handed to the caller. (Without a monitor, a state of at
+ * most 13 qubits runs all its blocks of one and two qubits in one pass; with
+ * one, they are split into passes of bounded arithmetic, as larger states'
+ * are.) The reference abandons by
  * throwing; across this ABI a nonzero return abandons instead: the state is
  * freed and the call returns MH_ERR_ABANDONED (the adapter rethrows what its
  * monitor threw). The next pass may already be queued when it runs, and is

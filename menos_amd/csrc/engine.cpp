@@ -67,12 +67,13 @@ double word_to_uniform(uint64_t w) { return static_cast<double>(w >> 11) * (1.0 
 // on the matrix cores for complex64 blocks of 5-6 qubits) takes the larger of
 // its HBM time and its arithmetic (8 * 2^k operations per amplitude and block) at the measured FP64 rate
 // (complex128, no FMA), twice that (complex64 FMA) or the matrix-core rate.
-double pass_seconds(uint32_t n, int32_t precision, const std::vector<Block>& blocks, uint32_t w, uint32_t max_cost) {
+double pass_seconds(uint32_t n, int32_t precision, const std::vector<Block>& blocks, uint32_t w, uint32_t max_cost,
+                    bool monitored = false) {
     const mh_calibration& c = g_calibration;
     const double sb = static_cast<double>(state_bytes(n, precision));
     const double amps = static_cast<double>(uint64_t{1} << n);
     double seconds = 0;
-    for (const WindowPass& pass : plan_window_passes(n, precision, blocks, w, max_cost)) {
+    for (const WindowPass& pass : plan_window_passes(n, precision, blocks, w, max_cost, monitored)) {
         if (!pass.generic) {
             seconds += 2.0 * sb / c.pass_bytes_per_second;
             continue;
@@ -184,7 +185,8 @@ CostEstimate HipDenseEngine::estimate(const ExecutionRequest& r) const noexcept 
         if (n > kMaxQubits) fail(MH_ERR_INVALID, "num_qubits above 40");
         const Plan p = make_plan(r);
         e.blocks = static_cast<uint32_t>(p.blocks.size());
-        e.passes = count_passes(n, r.precision, p.blocks, r.window_qubits, r.max_pass_cost);
+        const bool monitored = r.monitor != nullptr;
+        e.passes = count_passes(n, r.precision, p.blocks, r.window_qubits, r.max_pass_cost, monitored);
         e.fusion_used = p.fusion_used;
         e.width_used = p.width_used;
         const uint64_t sb = state_bytes(n, r.precision);
@@ -204,7 +206,7 @@ CostEstimate HipDenseEngine::estimate(const ExecutionRequest& r) const noexcept 
         double seconds = static_cast<double>(e.launches) * c.launch_seconds;
         seconds += n < window_default(r.precision)
                        ? static_cast<double>(e.passes) * 2.0 * static_cast<double>(sb) / c.pass_bytes_per_second
-                       : pass_seconds(n, r.precision, p.blocks, r.window_qubits, r.max_pass_cost);
+                       : pass_seconds(n, r.precision, p.blocks, r.window_qubits, r.max_pass_cost, monitored);
         seconds += static_cast<double>(sb) / c.hbm_bytes_per_second;  // initialisation
         seconds += (r.shots ? 3.0 : 0.0) * static_cast<double>(sb) / c.hbm_bytes_per_second;
         seconds += static_cast<double>(r.terms.size()) * static_cast<double>(sb) / c.hbm_bytes_per_second;

@@ -352,8 +352,8 @@ void apply_blocks(void* state, uint32_t n, int32_t precision, const std::vector<
 uint32_t window_default(int32_t precision) noexcept { return window_width(precision); }
 
 uint32_t count_passes(uint32_t n, int32_t precision, const std::vector<Block>& blocks, uint32_t window_qubits,
-                      uint32_t max_cost) {
-    return static_cast<uint32_t>(plan_window_passes(n, precision, blocks, window_qubits, max_cost).size());
+                      uint32_t max_cost, bool monitored) {
+    return static_cast<uint32_t>(plan_window_passes(n, precision, blocks, window_qubits, max_cost, monitored).size());
 }
 
 void launch_generic(void* state, uint32_t n, int32_t precision, const cplx* matrix, const uint32_t* operands,

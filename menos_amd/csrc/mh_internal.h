@@ -162,7 +162,7 @@ uint32_t window_default(int32_t precision) noexcept;
 
 // Number of HBM passes the schedule makes for these blocks.
 uint32_t count_passes(uint32_t n, int32_t precision, const std::vector<Block>& blocks, uint32_t window_qubits,
-                      uint32_t max_cost);
+                      uint32_t max_cost, bool monitored = false);
 
 bool matrix_is_diagonal(const cplx* m, std::size_t dim);
 
