@@ -310,7 +310,7 @@ typedef struct mh_cost_estimate {
     uint64_t work_units;     /* 2^n + sum over blocks 2^(n+k) + outputs (dense_engine.cpp:309-331) */
     uint32_t blocks;
     uint32_t passes;         /* HBM passes of the window schedule */
-    uint64_t launches;
+    uint64_t launches;       /* kernels, and the copy of the passes' tables or the initialisation */
     uint64_t h2d_bytes;
     uint64_t d2h_bytes;
     double seconds;          /* the calibrated time model's prediction */
@@ -324,7 +324,9 @@ typedef struct mh_cost_estimate {
  * are the calibrated profile's:
  *   launches * launch_seconds + passes * 2 * state / pass_bytes_per_second
  *   + state / hbm (initialisation) + 3 * state / hbm if sampling
- *   + terms * state / hbm + h2d / h2d_rate + d2h / d2h_rate. */
+ *   + terms * state / hbm + h2d / h2d_rate + d2h / d2h_rate
+ * (an upper bound for the outputs: the first window pass generates the state,
+ * sampling reads it about once, terms that share a tile set read it once). */
 int mh_engine_estimate(const mh_execution_request* request, mh_cost_estimate* out);
 int mh_engine_execute(const mh_execution_request* request, mh_execution_result* result);
 

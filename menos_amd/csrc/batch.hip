@@ -141,7 +141,7 @@ void EarlyReductions::queue(Bucket& b) {
     }
     b.program->launch_on(b.workspace.get(), reduce_, out_);
     b.queued = true;
-    launches_ += 2;
+    launches_ += b.program->launches();
 }
 
 void EarlyReductions::after(const BatchLaunch& l, hipStream_t stream) {
@@ -305,7 +305,7 @@ void execute_round(int32_t precision, std::vector<RoundItem>& items, uint32_t th
             const Counts counts = sample_counts(passes[k].state, it.n, precision, it.shots, it.seed,
                                                 it.targets ? *it.targets : kNone);
             *it.counts = std::map<uint64_t, uint64_t>(counts.begin(), counts.end());
-            launches += 7;
+            launches += sampler_launches(it.n);
         }
         if (it.statevector) download(it.statevector, passes[k].state, (uint64_t{1} << it.n) * amp);
     }

@@ -10,6 +10,7 @@
 // sampler.hip) instead of a copy-back and a host walk.
 #include "engine.hpp"
 #include "gate_table.h"
+#include "wide.h"
 #include "window.h"
 
 #include <algorithm>
@@ -40,14 +41,16 @@ constexpr uint32_t kMaxQubits = 40;
 
 uint64_t state_bytes(uint32_t n, int32_t precision) { return (uint64_t{1} << n) * amp_bytes(precision); }
 
-// Device scratch beside the state: the expectation partials and the sampler's
-// per-block tables (sampler.hip: 2^(n-13) blocks of about 100 bytes).
-uint64_t scratch_bytes(uint32_t n, uint64_t shots, std::size_t terms) {
-    uint64_t bytes = 0;
+// Device scratch beside the state: one pass's tables of wide blocks, or the
+// expectation partials, or the sampler's per-block tables (of states above 20
+// qubits an allowance of 112 bytes for each 2^13 amplitudes, about twice them).
+uint64_t scratch_bytes(uint32_t n, int32_t precision, const std::vector<Block>& blocks, uint64_t shots,
+                       std::size_t terms) {
+    uint64_t bytes = wide_pass_bytes(precision, n, blocks);
     if (terms) bytes = std::max<uint64_t>(bytes, 2048ull * 16 * 16 + 4096);
     if (shots) {
-        const uint64_t blocks = n > 13 ? (uint64_t{1} << (n - 13)) : 1;
-        bytes = std::max<uint64_t>(bytes, blocks * 112 + shots * 16 + 4096);
+        const uint64_t tables = std::max<uint64_t>(n > 13 ? (uint64_t{1} << (n - 13)) * 112 : 112, sampler_table_bytes(n));
+        bytes = std::max<uint64_t>(bytes, tables + shots * 16 + 4096);
     }
     return bytes + (64ull << 10);  // pass programs
 }
@@ -190,7 +193,7 @@ CostEstimate HipDenseEngine::estimate(const ExecutionRequest& r) const noexcept 
         e.fusion_used = p.fusion_used;
         e.width_used = p.width_used;
         const uint64_t sb = state_bytes(n, r.precision);
-        e.device_bytes = sb + scratch_bytes(n, r.shots, r.terms.size());
+        e.device_bytes = sb + scratch_bytes(n, r.precision, p.blocks, r.shots, r.terms.size());
         e.host_bytes = r.want_statevector ? sb : 0;
         // Work units as the reference counts them (dense_engine.cpp:309-331).
         uint64_t work = uint64_t{1} << n;
@@ -199,7 +202,12 @@ CostEstimate HipDenseEngine::estimate(const ExecutionRequest& r) const noexcept 
         if (r.shots) work += uint64_t{1} << n;
         work += r.terms.size() * (uint64_t{1} << n);
         e.work_units = work;
-        e.launches = 1 + e.passes + (r.shots ? 7 : 0) + 2 * r.terms.size();
+        // The first: the copy of the passes' tables, or the initialisation where
+        // no window pass generates the state.
+        std::vector<uint64_t> x;
+        for (const auto& t : r.terms) x.push_back(t.first);
+        e.launches = 1 + e.passes + (r.shots ? sampler_launches(n) : 0) +
+                     expectation_launches(n, x.data(), static_cast<uint32_t>(x.size()));
         e.h2d_bytes = 4096 + r.shots * 8;
         e.d2h_bytes = (r.want_statevector ? sb : 0) + r.shots * 8 + r.terms.size() * 16;
         const mh_calibration& c = g_calibration;
@@ -245,7 +253,7 @@ ExecutionResult HipDenseEngine::execute(const ExecutionRequest& r) const {
     DeviceLedger& ledger = DeviceLedger::current();
     ledger.reset();
     const uint64_t sb = state_bytes(n, r.precision);
-    const uint64_t need = sb + scratch_bytes(n, r.shots, r.terms.size());
+    const uint64_t need = sb + scratch_bytes(n, r.precision, p.blocks, r.shots, r.terms.size());
     if (r.budget_bytes != 0 && need > r.budget_bytes)
         fail(MH_ERR_RESOURCE, "the dense state needs " + std::to_string(need) + " device bytes, budget is " +
                                   std::to_string(r.budget_bytes));
@@ -278,6 +286,8 @@ ExecutionResult HipDenseEngine::execute(const ExecutionRequest& r) const {
             void* const data = r.monitor_data;
             stats.monitor = [fn, data](uint64_t crossed) { return fn(data, crossed) != 0; };
         }
+        if (r.budget_bytes != 0)
+            stats.wide_table_bytes = std::max<uint64_t>(1, std::min(kWideTableBytes, r.budget_bytes - need));
         apply_blocks(state.get(), n, r.precision, p.blocks, r.window_qubits, r.record_pass_times, &stats,
                      r.max_pass_cost, &phase);
         MH_HIP(hipEventRecord(g1, streams().main));

@@ -469,7 +469,32 @@ uint32_t blocks_for(uint64_t pairs) {
     return static_cast<uint32_t>(std::min<uint64_t>(kMaxBlocks, std::max<uint64_t>(1, pairs / (kThreads * 16))));
 }
 
+// The lowest qubits, which every tile holds.
+uint64_t tile_low(uint32_t n) { return (uint64_t{1} << std::min<uint32_t>(3, n)) - 1; }
+
+// How many bits the X mask of a tiled term may have, with the low run: the
+// tile's, but all twelve only where its partial sums (room for them: `share` of
+// four tiles each) then take no more room than the per-mask kernel's would (up to
+// 25 qubits).
+uint32_t tile_reach(uint32_t n, uint32_t share) {
+    const uint32_t k = std::min<uint32_t>(kTileBits, n);
+    return share <= blocks_for(uint64_t{1} << (n - 1)) ? k : std::min<uint32_t>(k, kTileBits - 1);
+}
+
+uint32_t tile_share(uint32_t n) {
+    return static_cast<uint32_t>(std::max<uint64_t>(1, (uint64_t{1} << (n - std::min<uint32_t>(kTileBits, n))) / 4));
+}
+
 }  // namespace
+
+uint32_t expectation_launches(uint32_t n, const uint64_t* x, uint32_t terms) {
+    if (terms == 0 || n == 0) return 0;
+    const uint32_t reach = tile_reach(n, tile_share(n));
+    bool tiled = false, wide = false;
+    for (uint32_t t = 0; t < terms; ++t)
+        (static_cast<uint32_t>(__builtin_popcountll(x[t] | tile_low(n))) > reach ? wide : tiled) = true;
+    return 1u + tiled + wide;
+}
 
 void expectation_terms(const void* state, uint32_t n, int32_t precision, const uint64_t* x, const uint64_t* z,
                        uint32_t terms, cplx* out) {
@@ -596,18 +621,15 @@ ExpPlan plan_expectation(const std::vector<ExpectationItem>& items) {
         const uintptr_t addr = reinterpret_cast<uintptr_t>(it.state);
         const uint64_t state_off = (addr - base_addr) / sizeof(V);
         const uint32_t k = std::min<uint32_t>(kTileBits, it.n);
-        const uint64_t low = (uint64_t{1} << std::min<uint32_t>(3, k)) - 1;
+        const uint64_t low = tile_low(it.n);
         // Sixteen tiles per workgroup of a large state, each workgroup a partial
         // sum per term (4.53 ms for 64 terms at 28 qubits; four tiles 4.98,
         // sixty-four 4.46 there but 2.42 against 2.36 for 24 terms). The room
         // set aside for partial sums is that of four tiles a workgroup: the
         // callers of the static workspace rely on what fits it.
         const uint32_t tiles = static_cast<uint32_t>(uint64_t{1} << (it.n - k));
-        const uint32_t share = std::max<uint32_t>(1, tiles / 4);
-        // A term is tiled if its X bits, with the low run, fit k tile bits; one
-        // that needs all twelve only if its partial sums then take no more
-        // room than the per-mask kernel's would.
-        const uint32_t reach = share <= blocks_for(uint64_t{1} << (it.n - 1)) ? k : std::min<uint32_t>(k, kTileBits - 1);
+        const uint32_t share = tile_share(it.n);
+        const uint32_t reach = tile_reach(it.n, share);
         std::vector<uint64_t> wide;
         std::vector<uint32_t> narrow;
         for (const auto& [xm, members] : groups) {
@@ -813,6 +835,11 @@ void ExpectationProgram::launch_on(void* workspace, hipStream_t stream, double* 
         launch_expectation<double2>(impl_->plan, workspace, stream, out);
     else
         launch_expectation<float2>(impl_->plan, workspace, stream, out);
+}
+
+uint32_t ExpectationProgram::launches() const {
+    const ExpPlan& p = impl_->plan;
+    return p.slots.empty() ? 0u : 1u + !p.tjobs.empty() + !p.jobs.empty();
 }
 
 void expectation_batch(int32_t precision, const std::vector<ExpectationItem>& items, double* out) {

@@ -146,6 +146,9 @@ struct PassStats {
     // Called after each completed pass with the passes completed so far;
     // true abandons (the queued work is waited for, then MH_ERR_ABANDONED).
     std::function<bool(uint64_t)> monitor;
+    // Device bytes for the tables of passes of wide blocks at a time (one pass's
+    // at least; 0: the default).
+    uint64_t wide_table_bytes = 0;
 };
 
 // Applies the blocks in order, grouped into window passes.
@@ -169,6 +172,9 @@ bool matrix_is_diagonal(const cplx* m, std::size_t dim);
 // ---- expectation (expectation.hip)
 void expectation_terms(const void* state, uint32_t n, int32_t precision, const uint64_t* x, const uint64_t* z,
                        uint32_t terms, cplx* out);
+
+// Its launches: the terms' tiles, the terms of wider X masks, what finishes both.
+uint32_t expectation_launches(uint32_t n, const uint64_t* x, uint32_t terms);
 
 // The terms of many states in two launches; results land at out[2 * (out_index + t)].
 struct ExpectationItem {
@@ -199,6 +205,7 @@ public:
     // waits: capturable); term t of item i lands at out[2 * (out_index + t)]
     // (device memory), or in the workspace's output region when out is null.
     void launch_on(void* workspace, hipStream_t stream, double* out = nullptr) const;
+    uint32_t launches() const;
 
 private:
     struct Impl;
@@ -208,6 +215,10 @@ private:
 // ---- sampler (sampler.hip)
 void sample_sorted(const void* state, uint32_t n, int32_t precision, const double* sorted_u, uint64_t shots,
                    uint64_t* basis_out);
+// Its launches for a state of n qubits, and the device bytes of its tables (none
+// of small states).
+uint32_t sampler_launches(uint32_t n);
+uint64_t sampler_table_bytes(uint32_t n);
 // Keeps `state` (2^n amplitudes) on the device with its sampler tables
 // (mh_region_sampler_*); synchronises.
 mh_region_sampler* make_region_sampler(DeviceBuffer&& state, uint32_t n, int32_t precision);

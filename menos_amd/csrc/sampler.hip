@@ -750,6 +750,16 @@ struct SamplerTables {
 
 uint64_t r16(uint64_t bytes) { return (bytes + 15) / 16 * 16; }
 
+uint64_t block_of(uint32_t n) {
+    return uint64_t{1} << std::min<uint32_t>(n, n <= kSmallBlockQubits ? kSmallBlockLog : kBlockLog);
+}
+
+uint64_t table_bytes(uint32_t n) {
+    const uint64_t nb = (uint64_t{1} << n) / block_of(n), groups = (nb + kGroup - 1) / kGroup;
+    return r16(nb * sizeof(Xfer)) + r16(groups * sizeof(Xfer)) + r16(nb * sizeof(double)) +
+           2 * r16((nb + 1) * sizeof(double)) + r16(groups * sizeof(double)) + r16(groups * sizeof(uint32_t));
+}
+
 // Allocates the tables of a state of 2^n amplitudes at `state`, or of such a
 // chunk of a state of `whole` qubits.
 void layout_tables(SamplerTables& t, const void* state, uint32_t n, uint32_t whole) {
@@ -757,13 +767,11 @@ void layout_tables(SamplerTables& t, const void* state, uint32_t n, uint32_t who
     SampleArgs& a = t.a;
     a.state = state;
     a.size = uint64_t{1} << n;
-    a.block = uint64_t{1} << std::min<uint32_t>(n, n <= kSmallBlockQubits ? kSmallBlockLog : kBlockLog);
+    a.block = block_of(n);
     a.blocks = static_cast<uint32_t>(a.size / a.block);
     a.groups = (a.blocks + kGroup - 1) / kGroup;
     const uint64_t nb = a.blocks;
-    t.buf = DeviceBuffer(r16(nb * sizeof(Xfer)) + r16(uint64_t(a.groups) * sizeof(Xfer)) + r16(nb * sizeof(double)) +
-                         2 * r16((nb + 1) * sizeof(double)) + r16(uint64_t(a.groups) * sizeof(double)) +
-                         r16(uint64_t(a.groups) * sizeof(uint32_t)));
+    t.buf = DeviceBuffer(table_bytes(n));
     char* p = t.buf.as<char>();
     auto take = [&](uint64_t bytes) {
         char* r = p;
@@ -934,6 +942,13 @@ void sample_sorted(const void* state, uint32_t n, int32_t precision, const doubl
     else
         run_sampler<float2>(state, n, sorted_u, shots, basis_out);
 }
+
+uint32_t sampler_launches(uint32_t n) {
+    if (n <= kSmallQubits) return 1;
+    return (uint64_t{1} << n) / block_of(n) > kGroup ? 8 : 7;
+}
+
+uint64_t sampler_table_bytes(uint32_t n) { return n <= kSmallQubits ? 0 : table_bytes(n); }
 
 struct ChunkedSampler::Impl {
     uint32_t n = 0, chunk_log = 0;

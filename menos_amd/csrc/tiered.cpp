@@ -157,8 +157,9 @@ struct TierRequest {
 uint64_t tier_scratch_bytes(uint32_t window, uint64_t shots, std::size_t terms) {
     uint64_t bytes = 64ull << 10;
     if (shots) {
-        const uint64_t blocks = window > 13 ? (uint64_t{1} << (window - 13)) : 1;
-        bytes += 2 * (blocks * 112 + 4096) + shots * 16 + 4096;
+        const uint64_t tables =
+            std::max<uint64_t>(window > 13 ? (uint64_t{1} << (window - 13)) * 112 : 112, sampler_table_bytes(window));
+        bytes += 2 * (tables + 4096) + shots * 16 + 4096;
     }
     if (terms) bytes += 2048ull * 16 * 16 + 4096;
     return bytes;

@@ -19,13 +19,16 @@ constexpr uint32_t kWideQubits = 34;
 // passes.
 constexpr uint32_t kWidePassBlocks = 16;
 
-// Tables of one upload, about.
+// Tables of one upload, about (a run with a budget keeps to what that leaves).
 constexpr uint64_t kWideTableBytes = uint64_t{16} << 20;
 
 // Whether a dense block of k qubits of an n-qubit state goes to a wide pass:
 // three to six qubits, except the complex64 blocks that the matrix cores take
 // and states beyond one launch.
 bool wide_applies(int32_t precision, uint32_t n, uint32_t k);
+
+// Device bytes of the tables of any one pass of these blocks, at most.
+uint64_t wide_pass_bytes(int32_t precision, uint32_t n, const std::vector<Block>& blocks);
 
 // The lowest qubits, which every tile holds: runs of 128 bytes.
 uint64_t wide_low_mask(int32_t precision);
@@ -42,6 +45,8 @@ public:
     // Returns the pass's index.
     uint32_t add(const std::vector<Block>& blocks, const std::vector<uint32_t>& which);
     uint64_t bytes() const;
+    // What add() would add to them, at most.
+    uint64_t bytes_of(const std::vector<Block>& blocks, const std::vector<uint32_t>& which) const;
     void upload();
     void launch(void* state, uint32_t pass, hipStream_t stream) const;
 

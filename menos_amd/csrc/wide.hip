@@ -224,6 +224,17 @@ bool wide_applies(int32_t precision, uint32_t n, uint32_t k) {
     return n >= kWideTileBits && n <= kWideQubits && k >= 3 && k <= (precision == MH_C128 ? kMaxK : 4);
 }
 
+uint64_t wide_pass_bytes(int32_t precision, uint32_t n, const std::vector<Block>& blocks) {
+    uint64_t sum = 0, most = 0;
+    for (const Block& b : blocks) {
+        if (b.diagonal || !wide_applies(precision, n, static_cast<uint32_t>(b.operands.size()))) continue;
+        const uint64_t bytes = sizeof(WideBlock) + b.matrix.size() * amp_bytes(precision);
+        sum += bytes;
+        most = std::max(most, bytes);
+    }
+    return sum == 0 ? 0 : std::min(sum, kWidePassBlocks * most) + 256;
+}
+
 uint64_t wide_low_mask(int32_t precision) { return precision == MH_C128 ? 7 : 15; }
 
 struct WidePasses::Impl {
@@ -324,6 +335,12 @@ uint32_t WidePasses::add(const std::vector<Block>& blocks, const std::vector<uin
     }
     d.passes.push_back(pass);
     return static_cast<uint32_t>(d.passes.size() - 1);
+}
+
+uint64_t WidePasses::bytes_of(const std::vector<Block>& blocks, const std::vector<uint32_t>& which) const {
+    uint64_t sum = 0;
+    for (uint32_t b : which) sum += sizeof(WideBlock) + blocks[b].matrix.size() * amp_bytes(impl_->precision);
+    return sum;
 }
 
 uint64_t WidePasses::bytes() const {
