@@ -42,8 +42,8 @@ __device__ __forceinline__ void load_amp(const V* s, uint64_t i, double& re, dou
     im = static_cast<double>(v.y);
 }
 
-// Workgroup `block` of `blocks` for one group of terms sharing an X mask:
-// writes partials[(t * blocks + block) * 2 + {0, 1}] for t < terms.
+// Workgroup `block` of `blocks` for one group of terms sharing an X mask (never
+// 0: diagonal terms fit any tile): writes partials[(t * blocks + block) * 2 + {0, 1}] for t < terms.
 template <typename V, uint32_t T>
 __device__ __forceinline__ void expectation_group(const V* s, double* partials, uint64_t pairs, uint64_t x, uint32_t h,
                                                   uint32_t terms, const uint64_t* z, uint32_t block, uint32_t blocks) {
@@ -59,61 +59,35 @@ __device__ __forceinline__ void expectation_group(const V* s, double* partials, 
     // before any is used (the loop is otherwise bound by memory latency), and
     // the sums still run over the items in order.
     constexpr uint32_t kUnroll = 4;
-    if (x == 0) {
-        for (uint64_t m0 = tid; m0 < pairs; m0 += kUnroll * total_threads) {
-            double ar[kUnroll], ai[kUnroll];
+    const uint64_t lowm = (1ull << h) - 1ull;
+    for (uint64_t r0 = tid; r0 < pairs; r0 += kUnroll * total_threads) {
+        double ar[kUnroll], ai[kUnroll], br[kUnroll], bi[kUnroll];
 #pragma unroll
-            for (uint32_t k = 0; k < kUnroll; ++k) {
-                const uint64_t m = m0 + k * total_threads;
-                if (m < pairs) load_amp(s, m, ar[k], ai[k]);
-            }
-#pragma unroll
-            for (uint32_t k = 0; k < kUnroll; ++k) {
-                const uint64_t m = m0 + k * total_threads;
-                if (m >= pairs) break;
-                // conj(a) * a: real ar*ar + ai*ai, imaginary ar*ai - ai*ar (exactly 0).
-                const double pr = ar[k] * ar[k] + ai[k] * ai[k];
-                const double pi = ar[k] * ai[k] - ai[k] * ar[k];
-#pragma unroll
-                for (uint32_t t = 0; t < T; ++t) {
-                    if (t >= terms) break;
-                    const bool neg = (__popcll(z[t] & m) & 1) != 0;
-                    accr[t] = neg ? accr[t] - pr : accr[t] + pr;
-                    acci[t] = neg ? acci[t] - pi : acci[t] + pi;
-                }
-            }
+        for (uint32_t k = 0; k < kUnroll; ++k) {
+            const uint64_t r = r0 + k * total_threads;
+            if (r >= pairs) continue;
+            const uint64_t m = ((r & ~lowm) << 1) | (r & lowm);
+            load_amp(s, m, ar[k], ai[k]);
+            load_amp(s, m ^ x, br[k], bi[k]);
         }
-    } else {
-        const uint64_t lowm = (1ull << h) - 1ull;
-        for (uint64_t r0 = tid; r0 < pairs; r0 += kUnroll * total_threads) {
-            double ar[kUnroll], ai[kUnroll], br[kUnroll], bi[kUnroll];
 #pragma unroll
-            for (uint32_t k = 0; k < kUnroll; ++k) {
-                const uint64_t r = r0 + k * total_threads;
-                if (r >= pairs) continue;
-                const uint64_t m = ((r & ~lowm) << 1) | (r & lowm);
-                load_amp(s, m, ar[k], ai[k]);
-                load_amp(s, m ^ x, br[k], bi[k]);
-            }
+        for (uint32_t k = 0; k < kUnroll; ++k) {
+            const uint64_t r = r0 + k * total_threads;
+            if (r >= pairs) break;
+            const uint64_t m = ((r & ~lowm) << 1) | (r & lowm);
+            const uint64_t mp = m ^ x;
+            // p = conj(a) * b
+            const double pr = ar[k] * br[k] + ai[k] * bi[k];
+            const double pi = ar[k] * bi[k] - ai[k] * br[k];
 #pragma unroll
-            for (uint32_t k = 0; k < kUnroll; ++k) {
-                const uint64_t r = r0 + k * total_threads;
-                if (r >= pairs) break;
-                const uint64_t m = ((r & ~lowm) << 1) | (r & lowm);
-                const uint64_t mp = m ^ x;
-                // p = conj(a) * b
-                const double pr = ar[k] * br[k] + ai[k] * bi[k];
-                const double pi = ar[k] * bi[k] - ai[k] * br[k];
-#pragma unroll
-                for (uint32_t t = 0; t < T; ++t) {
-                    if (t >= terms) break;
-                    const bool neg_mp = (__popcll(z[t] & mp) & 1) != 0;  // s(m') for p
-                    const bool neg_m = (__popcll(z[t] & m) & 1) != 0;    // s(m) for conj(p)
-                    accr[t] = neg_mp ? accr[t] - pr : accr[t] + pr;
-                    acci[t] = neg_mp ? acci[t] - pi : acci[t] + pi;
-                    accr[t] = neg_m ? accr[t] - pr : accr[t] + pr;
-                    acci[t] = neg_m ? acci[t] + pi : acci[t] - pi;
-                }
+            for (uint32_t t = 0; t < T; ++t) {
+                if (t >= terms) break;
+                const bool neg_mp = (__popcll(z[t] & mp) & 1) != 0;  // s(m') for p
+                const bool neg_m = (__popcll(z[t] & m) & 1) != 0;    // s(m) for conj(p)
+                accr[t] = neg_mp ? accr[t] - pr : accr[t] + pr;
+                acci[t] = neg_mp ? acci[t] - pi : acci[t] + pi;
+                accr[t] = neg_m ? accr[t] - pr : accr[t] + pr;
+                acci[t] = neg_m ? acci[t] + pi : acci[t] - pi;
             }
         }
     }
@@ -580,8 +554,8 @@ std::vector<std::vector<uint32_t>> pack_sets(const uint64_t* x, std::vector<uint
 
 // Plans every item's terms: X masks whose bits fit a tile (with the lowest
 // qubits) reduce from LDS tiles, a set of them per state read; any other X
-// mask (more than nine bits above qubit 2) takes the per-mask kernel; then one
-// finishing launch runs over every term.
+// mask (tile_reach) takes the per-mask kernel; then one finishing launch runs
+// over every term.
 template <typename V>
 ExpPlan plan_expectation(const std::vector<ExpectationItem>& items) {
     ExpPlan P;
