@@ -89,8 +89,13 @@ int mh_state_init(void* state, uint32_t num_qubits, int32_t precision, double ph
 /* One gate: a 2^k x 2^k matrix (host memory, 2*4^k doubles) at `operands`
  * (host memory), k <= 6, as one HBM pass. Diagonal blocks and blocks of 1 or 2
  * qubits run in the window-pass kernel (register windows, sign and diagonal
- * stages, controlled pairs), wider dense blocks in the per-group kernel; every
- * path is bitwise the generic kernel. */
+ * stages, controlled pairs, exact permutations as index maps), wider dense
+ * blocks on LDS tiles of states of 12 to 34 qubits (complex64 of 5 and 6 qubits
+ * on the matrix cores), else in the per-group kernel. On finite amplitudes every
+ * complex128 path is bitwise the generic kernel. Where an amplitude is infinite
+ * or NaN, which amplitudes of its groups are so afterwards depends on the path
+ * (a permutation may move it alone, products by zero may be left out); no other
+ * amplitude is affected. */
 int mh_apply_matrix(void* state, uint32_t num_qubits, int32_t precision, const double* matrix,
                     const uint32_t* operands, uint32_t k);
 

@@ -134,7 +134,7 @@ __device__ __forceinline__ void apply(unsigned char* lds, BlockPtr blk, EntryPtr
 // A block that permutes the basis (a Toffoli, a controlled SWAP): its sums are
 // one product by 1 and products by 0, so an output is its source plus the sum
 // of every input times zero: +0 where they are finite; where one is not, the
-// group turns NaN, as the sums would. Beside 8 * 2^k operations an amplitude it
+// group turns NaN, as its sums would (but for the part of an infinity moved). Beside 8 * 2^k operations an amplitude it
 // costs nothing: 24 blocks at 25 qubits, half of them Toffolis, 3.10 -> 2.55 ms.
 template <typename R, uint32_t K>
 __device__ __forceinline__ void permute(unsigned char* lds, BlockPtr blk, uint32_t t) {
