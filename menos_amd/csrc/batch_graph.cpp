@@ -457,6 +457,7 @@ void update_blocks(mh_batch_graph& gr, const mh_circuit* circuits, const double*
     set_phases(items, global_phases);
     const auto c0 = clock_type::now();
     BatchProgram prog = compile_batch_program(g->precision, items.data(), g->count, g->threads, g->schedule);
+    g->compile_seconds = seconds_since(c0);
     if (again) {
         g->captured = capture(*g, items, std::move(prog));
     } else {
@@ -464,7 +465,6 @@ void update_blocks(mh_batch_graph& gr, const mh_circuit* circuits, const double*
         std::memcpy(g->captured->pinned_mats.get(), prog.mats().data(), prog.mats().size());
         g->captured->program = std::move(prog);
     }
-    g->compile_seconds = seconds_since(c0);
     g->blocks = std::move(fresh);
     for (uint32_t i = 0; i < g->count; ++i)
         if (!wider[i].empty()) g->forms[i] = std::move(wider[i]);
